@@ -151,6 +151,49 @@ size_t join_generic_ws_bytes(int B);
 // largest power-of-two bucket count within it (cap_buckets).
 int join_table_capacity(int key_bytes);
 
+// ---------------------------------------------------------------------------
+// The plain join's own pipeline (pj_wide.h).
+// ---------------------------------------------------------------------------
+constexpr int kWideScan = 256;                     // digits per block of k_wide_scan
+constexpr int kWideScanMax = kMaxRadix / kWideScan;  // its blocks, at most
+
+// Index 0: build table, 1: probe table.
+struct WideArgs {
+  const void* keys[2];
+  const int32_t* pay[2];   // or nullptr (row ids)
+  void* tup[2];            // partitioned tuples
+  uint32_t n[2];
+  int bits;                // partitions: 2^bits; 0: none, the join reads the columns
+  uint32_t cap;            // build tuples per join chunk, at most
+  uint32_t slice;          // probe tuples per join item, at most
+  uint32_t tile;           // rows per scatter tile
+  uint32_t* cnt;           // [2][8][P] digit counts per XCD share, then write cursors
+  uint32_t* start[2];      // [P] partition starts relative to their scan block
+  uint32_t* iscan;         // [P rounded up to kWideScan] items before each partition, in its scan block
+  uint32_t* bsum;          // [3][kWideScanMax] block totals: build rows, probe rows, items
+  pj_pair* out;
+  uint64_t capacity;
+  unsigned long long* d_count;
+  int unique;              // a probe takes its first match only
+};
+
+struct WideShape {
+  int bits, cfg;           // partitions, join configuration
+  uint32_t cap, slice;
+  int rows_per_thread;     // of a scatter tile
+};
+
+// The pipeline's shape for tables of these sizes; false: more build rows than
+// one pass can split into chunks that fit the LDS.
+bool wide_shape(int64_t nR, int64_t nS, int key_bytes, WideShape* W);
+size_t wide_ws_bytes(int64_t nR, int64_t nS, int key_bytes, const WideShape& W);
+// Buffers from ws on; the counters, which a fill clears, end at `end`.
+void wide_carve(int64_t nR, int64_t nS, int key_bytes, const WideShape& W, char* ws, char* end, WideArgs* A);
+hipError_t launch_wide_hist(const WideArgs& A, int key_bytes, hipStream_t s);
+hipError_t launch_wide_scan(const WideArgs& A, hipStream_t s);
+hipError_t launch_wide_scatter(const WideArgs& A, int key_bytes, hipStream_t s);
+hipError_t launch_wide_join(const WideArgs& A, int key_bytes, int cfg, hipStream_t s);
+
 // log2 of the bucket count of the table of a build chunk of c tuples: the
 // power of two giving at least 4c slots (occupancy <= 1/4), at most
 // cap_buckets.  bs = slots per bucket.  A chunk is at most table_cap / 2 - 1

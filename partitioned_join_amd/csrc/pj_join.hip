@@ -36,6 +36,7 @@
 //                is dense in [0, total).
 #include "pj_device.h"
 #include "pj_internal.h"
+#include "pj_wide.h"
 
 
 namespace pj {
