@@ -167,10 +167,11 @@ struct WideArgs {
   uint32_t cap;            // build tuples per join chunk, at most
   uint32_t slice;          // probe tuples per join item, at most
   uint32_t tile;           // rows per scatter tile
+  uint32_t pad[2];         // free rows after each partition
   uint32_t* cnt;           // [2][8][P] digit counts per XCD share, then write cursors
   uint32_t* start[2];      // [P] partition starts relative to their scan block
   uint32_t* iscan;         // [P rounded up to kWideScan] items before each partition, in its scan block
-  uint32_t* bsum;          // [3][kWideScanMax] block totals: build rows, probe rows, items
+  uint32_t* bsum;          // [3][kWideScanMax] block totals: build rows, probe rows, items; then the items taken
   pj_pair* out;
   uint64_t capacity;
   unsigned long long* d_count;

@@ -73,6 +73,15 @@ __device__ __forceinline__ void pin(uint32_t& v) { __asm__ volatile("" : "+v"(v)
 __device__ __forceinline__ void pin(uint64_t& v) { __asm__ volatile("" : "+v"(v)); }
 __device__ __forceinline__ void pin(int32_t& v) { __asm__ volatile("" : "+v"(v)); }
 
+// The thread index through an opaque move, once per phase: row numbers formed
+// from it are then computed where they are used instead of being kept in
+// registers, which run out.
+__device__ __forceinline__ uint32_t opaque_tid() {
+  uint32_t t;
+  __asm__ volatile("v_mov_b32 %0, %1" : "=v"(t) : "v"(uint32_t(threadIdx.x)));
+  return t;
+}
+
 constexpr int kWideBlock = 1024;  // histogram and scatter workgroup
 
 // ---------------------------------------------------------------------------
@@ -176,7 +185,7 @@ __global__ __launch_bounds__(kWideScan) void k_wide_scan(WideArgs A) {
       sum += c[x];
     }
     tot[t] = sum;
-    uint32_t run = block_exclusive_scan<kWideScan>(sum, s_tmp[t], &total);
+    uint32_t run = block_exclusive_scan<kWideScan>(d < P ? sum + A.pad[t] : 0u, s_tmp[t], &total);
     if (d < P) {
       A.start[t][d] = run;
 #pragma unroll
@@ -193,7 +202,10 @@ __global__ __launch_bounds__(kWideScan) void k_wide_scan(WideArgs A) {
   A.iscan[d] = run;  // kWideScan entries per block, whatever P
   if (threadIdx.x == 0) {
     A.bsum[2 * kWideScanMax + blockIdx.x] = total;
-    if (blockIdx.x == 0) *A.d_count = 0ull;
+    if (blockIdx.x == 0) {
+      A.bsum[3 * kWideScanMax] = 0;  // the join's item tickets
+      *A.d_count = 0ull;
+    }
   }
 }
 
@@ -232,27 +244,29 @@ __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(4)))
   __shared__ uint32_t s_pre[3][kWideScanMax + 1];
   V* s_stage = reinterpret_cast<V*>(s_raw);
   const uint32_t P = 1u << A.bits, W = P / 2;
-  const int bits = A.bits;
+  const int shift = 32 - A.bits;  // at most 31: there is a digit
   uint32_t* s_cnt = reinterpret_cast<uint32_t*>(s_raw + size_t(TILE) * sizeof(V));  // W words: counts, then stage starts
   uint32_t* s_delta = s_cnt + W;                                                    // P words: output minus stage position
-  const uint32_t tid = threadIdx.x, wave = tid / kWave;
+  const uint32_t wave = sgpr(threadIdx.x / kWave);
   const uint32_t x = blockIdx.x % kNumXcd, G = gridDim.x;  // G is a multiple of 8
   const uint32_t nt0 = (A.n[0] + TILE - 1) / TILE, nt0r = (nt0 + kNumXcd - 1) / kNumXcd * kNumXcd;
   const uint32_t nt1 = (A.n[1] + TILE - 1) / TILE;
   const uint32_t nt = nt0r + nt1;  // tiles [nt0, nt0r) are empty, so that a tile's share is its index modulo 8
   block_prefixes(A, s_pre);
-  for (uint32_t i = tid; i < W; i += BLOCK) s_cnt[i] = 0;
+  for (uint32_t i = threadIdx.x; i < W; i += BLOCK) s_cnt[i] = 0;
 
   key_t key[E];
   int32_t pay[E];
   auto load = [&](uint32_t t) {
     const uint32_t tb = t >= nt0r ? 1u : 0u, n = A.n[tb], lo = (t - (tb ? nt0r : 0u)) * TILE;
-    const key_t* keys = static_cast<const key_t*>(A.keys[tb]);
+    const uint32_t tid = opaque_tid(), last = n - lo - 1u;
+    const key_t* keys = static_cast<const key_t*>(A.keys[tb]) + lo;  // a scalar row start and 32-bit lane offsets
 #pragma unroll
-    for (int e = 0; e < E; ++e) key[e] = __builtin_nontemporal_load(keys + min(lo + e * BLOCK + tid, n - 1));
+    for (int e = 0; e < E; ++e) key[e] = __builtin_nontemporal_load(keys + min(uint32_t(e) * BLOCK + tid, last));
     if (PAY && A.pay[tb]) {
+      const int32_t* p = A.pay[tb] + lo;
 #pragma unroll
-      for (int e = 0; e < E; ++e) pay[e] = __builtin_nontemporal_load(A.pay[tb] + min(lo + e * BLOCK + tid, n - 1));
+      for (int e = 0; e < E; ++e) pay[e] = __builtin_nontemporal_load(p + min(uint32_t(e) * BLOCK + tid, last));
     }
   };
   auto next_tile = [&](uint32_t t) {
@@ -266,24 +280,25 @@ __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(4)))
   while (t < nt) {
     const uint32_t tb = t >= nt0r ? 1u : 0u, n = A.n[tb], lo = (t - (tb ? nt0r : 0u)) * TILE;
     const uint32_t len = min(TILE, n - lo);
-    uint32_t* cursor = A.cnt + size_t(tb * kNumXcd + x) * P;
+    unsigned long long* cursor = reinterpret_cast<unsigned long long*>(A.cnt + size_t(tb * kNumXcd + x) * P);
     // digit << 16 | rank within it
     uint32_t pk[E];
     {
-      const uint32_t d0 = top_bits(wide_hash(key[0]), bits);
+      const uint32_t tid = opaque_tid();
+      const uint32_t d0 = wide_hash(key[0]) >> shift;
       // same-address LDS adds serialise: under a heavy key each row's lanes
       // with lane 0's digit rank with one add
       const bool heavy = __popcll(__ballot(d0 == sgpr(d0))) >= kHeavyLanes;
       if (!heavy && len == TILE) {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-          const uint32_t d = top_bits(wide_hash(key[e]), bits), sh = (d & 1u) << 4;
+          const uint32_t d = wide_hash(key[e]) >> shift, sh = (d & 1u) << 4;
           pk[e] = (d << 16) | ((atomicAdd(&s_cnt[d >> 1], 1u << sh) >> sh) & 0xFFFFu);
         }
       } else {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-          const uint32_t d = top_bits(wide_hash(key[e]), bits), sh = (d & 1u) << 4;
+          const uint32_t d = wide_hash(key[e]) >> shift, sh = (d & 1u) << 4;
           const bool valid = e * BLOCK + tid < len;
           const uint32_t f = sgpr(d);
           const uint64_t same = __ballot(valid && d == f);
@@ -300,8 +315,13 @@ __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(4)))
       }
     }
     lds_barrier();
-    // stage and output ranges of this thread's digits, 2 per count word
-    uint32_t c[WPT], g0[WPT], g1[WPT], mine = 0;
+    // Stage and output ranges of this thread's digits, 2 per count word.  The
+    // two digits' cursors advance in one 64-bit add (a cursor stays below
+    // 2^32, so nothing carries into the second): every line of cursors an add
+    // touches is written through to memory, half the adds write half as much.
+    const uint32_t tid = opaque_tid();
+    uint32_t c[WPT], mine = 0;
+    unsigned long long g[WPT];
 #pragma unroll
     for (int k = 0; k < WPT; ++k) {
       c[k] = tid + k * BLOCK < W ? s_cnt[tid + k * BLOCK] : 0u;
@@ -309,30 +329,28 @@ __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(4)))
     }
 #pragma unroll
     for (int k = 0; k < WPT; ++k) {
-      const uint32_t d = 2u * (tid + k * BLOCK);
-      g0[k] = g1[k] = 0;
-      if (c[k] & 0xFFFFu) g0[k] = atomicAdd(&cursor[d], c[k] & 0xFFFFu);
-      if (c[k] >> 16) g1[k] = atomicAdd(&cursor[d + 1], c[k] >> 16);
+      g[k] = 0;
+      if (c[k]) g[k] = atomicAdd(cursor + tid + k * BLOCK, (unsigned long long)(c[k] & 0xFFFFu) | ((unsigned long long)(c[k] >> 16) << 32));
     }
     const uint32_t inc = wave_scan(mine);
     if ((tid & (kWave - 1)) == kWave - 1) s_wsum[wave] = inc;
     lds_barrier();
     uint32_t run = inc - mine;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) run += w < int(wave) ? s_wsum[w] : 0u;
+    for (int w = 0; w < NW; ++w) run += w < int(wave) ? sgpr(s_wsum[w]) : 0u;
 #pragma unroll
     for (int k = 0; k < WPT; ++k)
       if (tid + k * BLOCK < W) {
-        const uint32_t a = c[k] & 0xFFFFu;
-        s_cnt[tid + k * BLOCK] = run | ((run + a) << 16);
-        g0[k] -= run;
-        g1[k] -= run + a;
-        run += a + (c[k] >> 16);
+        const uint32_t a = c[k] & 0xFFFFu, b = c[k] >> 16;
+        c[k] = run | ((run + a) << 16);
+        s_cnt[tid + k * BLOCK] = c[k];
+        run += a + b;
       }
     lds_barrier();
+    const uint32_t tid_s = opaque_tid();
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      const uint32_t i = e * BLOCK + tid;
+      const uint32_t i = e * BLOCK + tid_s;
       if (i < len) {
         const uint32_t d = pk[e] >> 16;
         const int32_t p = PAY && A.pay[tb] ? pay[e] : int32_t(lo + i);
@@ -343,8 +361,8 @@ __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(4)))
     for (int k = 0; k < WPT; ++k)
       if (tid + k * BLOCK < W) {
         const uint32_t d = 2u * (tid + k * BLOCK), pre = s_pre[tb][d / kWideScan];
-        s_delta[d] = g0[k] + pre;
-        s_delta[d + 1] = g1[k] + pre;
+        s_delta[d] = uint32_t(g[k]) + pre - (c[k] & 0xFFFFu);
+        s_delta[d + 1] = uint32_t(g[k] >> 32) + pre - (c[k] >> 16);
       }
     // the next tile's loads are in flight during the flush (the last tile's
     // are read again rather than branch)
@@ -355,22 +373,24 @@ __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(4)))
     // of a full tile unconditional, so that the next wait for the loads does
     // not wait for them.
     V* out = static_cast<V*>(A.tup[tb]);
+    const uint32_t end = n + P * A.pad[tb] - 1u;
+    const uint32_t tid_f = opaque_tid();
     if (len == TILE) {
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-        const uint32_t q = e * BLOCK + tid;
+        const uint32_t q = e * BLOCK + tid_f;
         const V v = s_stage[q];
-        const uint32_t p = s_delta[top_bits(wide_hash(WideTup<KB>::key(v)), bits)] + q;
-        out[min(p, n - 1)] = v;
+        const uint32_t p = s_delta[wide_hash(WideTup<KB>::key(v)) >> shift] + q;
+        out[min(p, end)] = v;
       }
     } else {
-      for (uint32_t q = tid; q < len; q += BLOCK) {
+      for (uint32_t q = tid_f; q < len; q += BLOCK) {
         const V v = s_stage[q];
-        const uint32_t p = s_delta[top_bits(wide_hash(WideTup<KB>::key(v)), bits)] + q;
-        out[min(p, n - 1)] = v;
+        const uint32_t p = s_delta[wide_hash(WideTup<KB>::key(v)) >> shift] + q;
+        out[min(p, end)] = v;
       }
     }
-    for (uint32_t i = tid; i < W; i += BLOCK) s_cnt[i] = 0;
+    for (uint32_t i = tid_f; i < W; i += BLOCK) s_cnt[i] = 0;
     lds_barrier();
     t = tn;
   }
@@ -379,6 +399,8 @@ __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(4)))
 // ---------------------------------------------------------------------------
 // k_wide_join
 // ---------------------------------------------------------------------------
+constexpr uint32_t kWideSpare = 8;
+
 struct WideItem {
   uint32_t rlo, rhi, slo, shi;
 };
@@ -416,26 +438,19 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
   constexpr int NW = BLOCK / kWave;
   constexpr uint32_t WPT = NBK / 2 / BLOCK;  // bucket words per thread
   static_assert(WPT >= 1 && WPT * BLOCK * 2 == NBK, "whole bucket words per thread");
-  static_assert(CAP < 65536 && CAP % 8 == 0, "bucket starts are 16-bit, arrays aligned");
+  static_assert(CAP < 65536 && CAP % 8 == 0 && kWideSpare % 4 == 0, "bucket starts are 16-bit, arrays aligned");
   static_assert(VERIFY || KB == 4, "8-byte keys are compared");
   extern __shared__ __align__(16) uint8_t s_raw[];
-  // keys (VERIFY), payloads, bucket starts (two to a word, and the end), tags (and spare bytes for the last window)
+  // keys (VERIFY), payloads, bucket starts (two to a word, and the end), tags; kWideSpare entries past the last one
   key_t* s_key = reinterpret_cast<key_t*>(s_raw);
-  int32_t* s_pay = reinterpret_cast<int32_t*>(s_raw + (VERIFY ? size_t(CAP) * KB : 0));
-  uint32_t* s_off = reinterpret_cast<uint32_t*>(s_pay + CAP);
+  int32_t* s_pay = reinterpret_cast<int32_t*>(s_raw + (VERIFY ? size_t(CAP + kWideSpare) * KB : 0));
+  uint32_t* s_off = reinterpret_cast<uint32_t*>(s_pay + CAP + kWideSpare);  // 16-byte aligned
   uint8_t* s_tag = reinterpret_cast<uint8_t*>(s_off + NBK / 2 + 2);
   __shared__ uint32_t s_wsum[NW];
   __shared__ uint32_t s_wtot[2][NW];
   __shared__ uint64_t s_base[2];
+  __shared__ uint32_t s_next;
   __shared__ uint32_t s_pre[3][kWideScanMax + 1];
-  // The thread index through an opaque move, per phase: row numbers formed
-  // from it are then computed where they are used instead of being kept in
-  // registers, which run out.
-  auto opaque_tid = [&]() {
-    uint32_t t;
-    __asm__ volatile("v_mov_b32 %0, %1" : "=v"(t) : "v"(uint32_t(threadIdx.x)));
-    return t;
-  };
   const uint32_t wave = sgpr(threadIdx.x / kWave);
   const int bits = COLS ? 0 : A.bits;
   const uint32_t grid = gridDim.x;
@@ -471,8 +486,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     const uint32_t first = sgpr(A.iscan[q]);
     const uint32_t r0 = sgpr(A.start[0][q]) + sgpr(s_pre[0][blk]), s0 = sgpr(A.start[1][q]) + sgpr(s_pre[1][blk]);
     const uint32_t qn = q + 1, bn = qn / kWideScan;
-    const uint32_t r1 = qn < P ? sgpr(A.start[0][qn]) + sgpr(s_pre[0][bn]) : A.n[0];
-    const uint32_t s1 = qn < P ? sgpr(A.start[1][qn]) + sgpr(s_pre[1][bn]) : A.n[1];
+    const uint32_t r1 = (qn < P ? sgpr(A.start[0][qn]) + sgpr(s_pre[0][bn]) : sgpr(s_pre[0][nblk])) - A.pad[0];
+    const uint32_t s1 = (qn < P ? sgpr(A.start[1][qn]) + sgpr(s_pre[1][bn]) : sgpr(s_pre[1][nblk])) - A.pad[1];
     const uint32_t ns = (s1 - s0 - 1) / A.slice + 1, k = local - first;
     w.rlo = r0 + (k / ns) * A.cap;
     w.rhi = min(r1, w.rlo + A.cap);
@@ -481,24 +496,20 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     return w;
   };
 
-  // Row k of a thread is lo + k * BLOCK + tid: rows wholly past the range's
-  // end are skipped (a uniform branch), lanes past it reread its last row.
-  // The row's start is a scalar, so that a lane's address is one 32-bit
-  // offset.  A row left alone is set to zero: it would otherwise keep its
-  // last value's registers through the probes.
+  // Row k of a thread is lo + k * BLOCK + tid; rows past the range's end read
+  // its last one again (one line for the whole wave) rather than branch: with
+  // a branch a row, the compiler moved each row's registers at the branch's
+  // end, which waits for its load (the build of 16384 tuples took 30 us).
+  // `lo` is a scalar, so that a lane's address is one 32-bit offset.
   auto load_row = [&](int side, uint32_t lo, uint32_t hi, uint32_t tid, key_t& k, int32_t& p) {
-    k = 0;
-    p = 0;
-    if (lo < hi) {
-      const uint32_t i = min(tid, hi - lo - 1u);
-      if constexpr (COLS) {
-        k = (static_cast<const key_t*>(A.keys[side]) + lo)[i];
-        p = A.pay[side] ? (A.pay[side] + lo)[i] : int32_t(lo + i);
-      } else {
-        const V v = (static_cast<const V*>(A.tup[side]) + lo)[i];
-        k = WideTup<KB>::key(v);
-        p = WideTup<KB>::pay(v);
-      }
+    const uint32_t i = min(lo + tid, hi - 1u);
+    if constexpr (COLS) {
+      k = static_cast<const key_t*>(A.keys[side])[i];
+      p = A.pay[side] ? A.pay[side][i] : int32_t(i);
+    } else {
+      const V v = static_cast<const V*>(A.tup[side])[i];
+      k = WideTup<KB>::key(v);
+      p = WideTup<KB>::pay(v);
     }
   };
   key_t bk[NB];
@@ -507,6 +518,17 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     const uint32_t tid = opaque_tid();
 #pragma unroll
     for (int k = 0; k < NB; ++k) load_row(0, w.rlo + uint32_t(k) * BLOCK, w.rhi, tid, bk[k], bp[k]);
+  };
+  // Brings the chunk's lines into the L2 while the last item's matches go out:
+  // one load of a word per line, whose value nobody reads.  (Loading the
+  // tuples themselves there costs twice the registers there are.)
+  auto touch_build = [&](const WideItem& w) {
+    if constexpr (!COLS) {
+      const char* at = static_cast<const char*>(A.tup[0]) + size_t(w.rlo) * sizeof(V);
+      const uint32_t bytes = (w.rhi - w.rlo) * uint32_t(sizeof(V));
+      for (uint32_t o = opaque_tid() * 128u; o < bytes; o += uint32_t(BLOCK) * 128u)
+        (void)*reinterpret_cast<const volatile uint32_t*>(at + o);
+    }
   };
   key_t pk[U], nk[U];
   int32_t pp[U], np[U];
@@ -532,14 +554,15 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
   uint32_t item = blockIdx.x;
   if (item >= total_items) return;
   WideItem w = decode(item);
-  load_build(w);
-  load_probe(w.slo, w.shi, pk, pp);
   uint32_t par = 0;  // parity of the round: which s_wtot / s_base slot
   while (true) {
     // ---- build
     const uint32_t c = w.rhi - w.rlo;
+    uint32_t ticket = 0;  // thread 0: the next item, taken now and read after the item's last round
     {
       const uint32_t tid = opaque_tid();
+      if (!COLS && tid == 0) ticket = grid + atomicAdd(A.bsum + 3 * kWideScanMax, 1u);
+      load_build(w);
 #pragma unroll
       for (uint32_t i = 0; i < WPT; ++i) s_off[tid + i * BLOCK] = 0;
       lds_barrier();
@@ -553,14 +576,25 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
           rk[k / 2] |= (k & 1) ? r << 16 : r;
         }
       }
+      // the first probe round is on its way during the scan and the writes
+      // (any earlier its registers are one too many)
+      load_probe(w.slo, w.shi, pk, pp);
       lds_barrier();
       {
+        // this thread's words, 16 bytes at a time where there are four
         uint32_t v[WPT], sum = 0;
+        if constexpr (WPT % 4 == 0) {
 #pragma unroll
-        for (uint32_t i = 0; i < WPT; ++i) {
-          v[i] = s_off[tid * WPT + i];
-          sum += (v[i] & 0xFFFFu) + (v[i] >> 16);
+          for (uint32_t i = 0; i < WPT / 4; ++i) {
+            const u32x4 q = reinterpret_cast<const u32x4*>(s_off)[tid * (WPT / 4) + i];
+            v[4 * i] = q.x; v[4 * i + 1] = q.y; v[4 * i + 2] = q.z; v[4 * i + 3] = q.w;
+          }
+        } else {
+#pragma unroll
+          for (uint32_t i = 0; i < WPT; ++i) v[i] = s_off[tid * WPT + i];
         }
+#pragma unroll
+        for (uint32_t i = 0; i < WPT; ++i) sum += (v[i] & 0xFFFFu) + (v[i] >> 16);
         const uint32_t inc = wave_scan(sum);
         if ((tid & (kWave - 1)) == kWave - 1) s_wsum[wave] = inc;
         lds_barrier();
@@ -569,9 +603,17 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         for (int i = 0; i < NW; ++i) run += i < int(wave) ? sgpr(s_wsum[i]) : 0u;
 #pragma unroll
         for (uint32_t i = 0; i < WPT; ++i) {
-          const uint32_t a = v[i] & 0xFFFFu;
-          s_off[tid * WPT + i] = run | ((run + a) << 16);
-          run += a + (v[i] >> 16);
+          const uint32_t a = v[i] & 0xFFFFu, b = v[i] >> 16;
+          v[i] = run | ((run + a) << 16);
+          run += a + b;
+        }
+        if constexpr (WPT % 4 == 0) {
+#pragma unroll
+          for (uint32_t i = 0; i < WPT / 4; ++i)
+            reinterpret_cast<u32x4*>(s_off)[tid * (WPT / 4) + i] = u32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+        } else {
+#pragma unroll
+          for (uint32_t i = 0; i < WPT; ++i) s_off[tid * WPT + i] = v[i];
         }
         if (tid == 0) s_off[NBK / 2] = c;
       }
@@ -590,7 +632,6 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     }
 
     // ---- probe
-    const uint32_t item_n = item + grid;
     bool pending = false;  // a round's matches are held, to be stored
     uint64_t h_m[U];       // its matches: a lane mask per probe row
     uint32_t h_pre = 0, h_n = 0;  // the pairs of the waves before this one, and of this wave
@@ -627,8 +668,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
       uint64_t m[U];
       int32_t fb[U];
 #pragma unroll
-      for (int k = 0; k < U; ++k)
-        bd[k] = r0 + uint32_t(k) * BLOCK + nlane < w.shi ? bounds_of(wide_hash(pk[k])) : 0u;
+      for (int k = 0; k < U; ++k) {
+        const uint32_t b = bounds_of(wide_hash(pk[k]));
+        bd[k] = r0 + uint32_t(k) * BLOCK + nlane < w.shi ? b : 0u;
+      }
 #pragma unroll
       for (int k = 0; k < U; ++k) {
         const uint32_t lo = bd[k] & 0xFFFFu, n = (bd[k] >> 16) - lo;
@@ -640,15 +683,15 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         // the first tag that fits; none: entry lo, unused
         fb[k] = int32_t(lo + (uint32_t(__builtin_ctz(z | 0x80000000u)) >> 3));
         bool hit = z != 0;
-        const bool again = n > 4u || (z & (z - 1u)) != 0;
-        slow |= again && !(first_only && !VERIFY && hit) ? 1u << k : 0u;
+        const bool again = (n > 4u) | ((z & (z - 1u)) != 0);
+        slow |= again & !(first_only & !VERIFY & hit) ? 1u << k : 0u;
         m[k] = __ballot(hit);
       }
       if constexpr (VERIFY) {
 #pragma unroll
         for (int k = 0; k < U; ++k) {
           const bool hit = (m[k] >> lane_id()) & 1u;
-          const bool same = hit && s_key[fb[k]] == pk[k];
+          const bool same = hit & (s_key[fb[k]] == pk[k]);
           // another tag may still fit, or the bucket go on past the window
           if (first_only && same) slow &= ~(1u << k);
           m[k] = __ballot(same);
@@ -691,7 +734,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         wtot = uint32_t(__builtin_amdgcn_readlane(int(inc), kWave - 1));
       }
       if (lane_id() == 0) s_wtot[par][wave] = wtot | (wave_multi ? 0x80000000u : 0u);
-      if (threadIdx.x == 0 && pending) s_base[par ^ 1] = claim;
+      if (threadIdx.x == 0) {
+        if (pending) s_base[par ^ 1] = claim;
+        if (!COLS && !more) s_next = ticket;
+      }
       lds_barrier();
       // every wave's pairs, in the lanes of each wave
       const uint32_t wt = lane_id() < uint32_t(NW) ? s_wtot[par][lane_id()] : 0u;
@@ -751,11 +797,11 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
       }
     }
     // ---- the next item's tuples are on their way while the last matches go out
+    const uint32_t item_n = COLS ? item + grid : sgpr(s_next);
     const bool last = item_n >= total_items;
     if (!last) {
       w = decode(item_n);
-      load_build(w);
-      load_probe(w.slo, w.shi, pk, pp);
+      touch_build(w);
     }
     if (threadIdx.x == 0 && pending) s_base[par ^ 1] = claim;
     lds_barrier();  // also: every wave is done with the table
@@ -778,7 +824,7 @@ struct WideCfg {
   bool verify;
   constexpr uint32_t cap() const { return uint32_t(block * nb); }
   constexpr size_t lds(int kb) const {
-    return size_t(cap()) * ((verify ? kb : 0) + 5) + (size_t(1) << lgb) * 2 + 8 + 16;
+    return size_t(cap() + kWideSpare) * ((verify ? kb : 0) + 5) + (size_t(1) << lgb) * 2 + 8;
   }
 };
 static constexpr WideCfg kWideCfg4[5] = {{512, 6, 11, true}, {512, 12, 13, true}, {512, 17, 13, false},
@@ -863,6 +909,8 @@ bool wide_shape(int64_t nR, int64_t nS, int key_bytes, WideShape* W) {
   const double chunk = n / double(1 << bits);
   double sl = 8.0 * chunk, fill = double(nS) / 1024.0;
   if (sl > fill) sl = fill > chunk ? fill : chunk;
+  // With enough partitions an ordinary one is one item.
+  if (bits >= 10 && sl < 1.25 * double(nS) / double(1 << bits)) sl = 1.25 * double(nS) / double(1 << bits);
   uint64_t slice = (uint64_t(sl) + round - 1) / round * round;
   if (slice < round) slice = round;
   W->slice = uint32_t(slice < (1u << 20) ? slice : (1u << 20));
@@ -874,12 +922,21 @@ bool wide_shape(int64_t nR, int64_t nS, int key_bytes, WideShape* W) {
   return true;
 }
 
+// Rows left free after each partition, so that partitions start an odd number
+// of 128-byte lines apart on average.
+static uint32_t wide_pad(int64_t n, int key_bytes, int bits) {
+  const uint32_t per_line = key_bytes == 4 ? 16 : 8;
+  const uint32_t lines = uint32_t((n >> bits) / per_line);
+  return (lines % 2 ? 4u : 5u) * per_line;
+}
+
 size_t wide_ws_bytes(int64_t nR, int64_t nS, int key_bytes, const WideShape& W) {
   if (W.bits == 0) return 0;
   auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
   const size_t P = size_t(1) << W.bits, tb = key_bytes == 4 ? 8 : 16;
   const size_t scan = (P + kWideScan - 1) / kWideScan * kWideScan;
-  return up(size_t(nR) * tb) + up(size_t(nS) * tb) + 2 * up(P * 4) + up(scan * 4) + up(3 * kWideScanMax * 4) +
+  return up((size_t(nR) + P * wide_pad(nR, key_bytes, W.bits)) * tb) +
+         up((size_t(nS) + P * wide_pad(nS, key_bytes, W.bits)) * tb) + 2 * up(P * 4) + up(scan * 4) + up((3 * kWideScanMax + 1) * 4) +
          up(2 * kNumXcd * P * 4);
 }
 
@@ -897,12 +954,14 @@ void wide_carve(int64_t nR, int64_t nS, int key_bytes, const WideShape& W, char*
     return p;
   };
   const size_t P = size_t(1) << W.bits, tb = key_bytes == 4 ? 8 : 16;
-  A->tup[0] = take(size_t(nR) * tb);
-  A->tup[1] = take(size_t(nS) * tb);
+  A->pad[0] = wide_pad(nR, key_bytes, W.bits);
+  A->pad[1] = wide_pad(nS, key_bytes, W.bits);
+  A->tup[0] = take((size_t(nR) + P * A->pad[0]) * tb);
+  A->tup[1] = take((size_t(nS) + P * A->pad[1]) * tb);
   A->start[0] = reinterpret_cast<uint32_t*>(take(P * 4));
   A->start[1] = reinterpret_cast<uint32_t*>(take(P * 4));
   A->iscan = reinterpret_cast<uint32_t*>(take((P + kWideScan - 1) / kWideScan * kWideScan * 4));
-  A->bsum = reinterpret_cast<uint32_t*>(take(3 * kWideScanMax * 4));
+  A->bsum = reinterpret_cast<uint32_t*>(take((3 * kWideScanMax + 1) * 4));
   A->cnt = reinterpret_cast<uint32_t*>(end - ((2 * kNumXcd * P * 4 + 255) & ~size_t(255)));  // the workspace's last bytes
 }
 
