@@ -178,37 +178,42 @@ hipError_t project_reference(const void* keys, int key_bytes, const pj_pair* pai
 // ---------------------------------------------------------------------------
 // Gather of payload columns through the join's pairs (cuDF's gather map):
 // out_build[i] = build_col[pairs[i].build_idx], out_probe[i] =
-// probe_col[pairs[i].probe_idx].  Each thread handles 4 pairs (two 16-byte
-// pair loads); the column reads are random and the writes coalesced.
+// probe_col[pairs[i].probe_idx].  The column reads are random, a 128-byte line
+// for each 4- or 8-byte element, and bound the kernel; the rest streams.  A
+// join's pairs come partition by partition, and a partition's pairs name the
+// same build rows again and again: so each XCD takes one contiguous eighth of
+// the pairs, and its workgroups walk it side by side, one pair a thread and
+// two workgroups per CU (16K pairs in flight), so that the lines of the
+// partition at hand stay in its L2 until they have been read again.  10M and
+// 40M rows, 40M pairs: 1.93 ms and 10.3 GB fetched with the pairs dealt over
+// all XCDs and 8192 workgroups, 0.93 ms and 6.7 GB here; 1.23 ms with 4 or 8
+// workgroups per CU, whose partitions in flight overflow the L2.
 // ---------------------------------------------------------------------------
+constexpr int kGatherBlock = 256;
+constexpr int kGatherGrid = 512;  // two per CU
+
 template <typename TB, typename TP>
-__global__ __launch_bounds__(256) void k_gather(const uint2* pairs, int64_t n, const TB* bcol, const TP* pcol,
-                                                TB* bout, TP* pout) {
-  const int64_t groups = (n + 3) / 4;
-  PJ_GRID_STRIDE(g, groups) {
-    const int64_t i0 = g * 4;
-    uint2 pr[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) pr[c] = i0 + c < n ? pairs[i0 + c] : make_uint2(0u, 0u);
-    TB vb[4];
-    TP vp[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      if (bcol && i0 + c < n) vb[c] = bcol[int32_t(pr[c].x)];
-      if (pcol && i0 + c < n) vp[c] = pcol[int32_t(pr[c].y)];
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      if (bcol && i0 + c < n) bout[i0 + c] = vb[c];
-      if (pcol && i0 + c < n) pout[i0 + c] = vp[c];
-    }
+__global__ __launch_bounds__(kGatherBlock) void k_gather(const uint2* pairs, int64_t n, const TB* bcol, const TP* pcol,
+                                                         TB* bout, TP* pout) {
+  const int64_t per = (n + kNumXcd * kGatherBlock - 1) / (kNumXcd * kGatherBlock) * kGatherBlock;  // pairs per XCD
+  const int64_t lo = int64_t(blockIdx.x % kNumXcd) * per, hi = n < lo + per ? n : lo + per;
+  const int64_t step = int64_t(gridDim.x / kNumXcd) * kGatherBlock;
+  for (int64_t i = lo + int64_t(blockIdx.x / kNumXcd) * kGatherBlock + threadIdx.x; i < hi; i += step) {
+    const unsigned long long pr = __builtin_nontemporal_load(reinterpret_cast<const unsigned long long*>(pairs) + i);
+    TB vb{};
+    TP vp{};
+    if (bcol) vb = bcol[int32_t(uint32_t(pr))];
+    if (pcol) vp = pcol[int32_t(uint32_t(pr >> 32))];
+    if (bcol) __builtin_nontemporal_store(vb, bout + i);
+    if (pcol) __builtin_nontemporal_store(vp, pout + i);
   }
 }
 
 template <typename TB, typename TP>
 static hipError_t gather_t(const pj_pair* pairs, int64_t n, const void* bcol, const void* pcol, void* bout,
                            void* pout, hipStream_t s) {
-  hipLaunchKernelGGL((k_gather<TB, TP>), dim3(grid_for((n + 3) / 4, 256)), dim3(256), 0, s,
+  const int64_t blocks = (n + kNumXcd * kGatherBlock - 1) / (kNumXcd * kGatherBlock) * kNumXcd;
+  hipLaunchKernelGGL((k_gather<TB, TP>), dim3(int(blocks < kGatherGrid ? blocks : kGatherGrid)), dim3(kGatherBlock), 0, s,
                      reinterpret_cast<const uint2*>(pairs), n, static_cast<const TB*>(bcol),
                      static_cast<const TP*>(pcol), static_cast<TB*>(bout), static_cast<TP*>(pout));
   return hipGetLastError();
