@@ -21,7 +21,7 @@ constexpr int kJoinProbe8 = 4;        // 8-byte keys (2048 per round)
 constexpr int kJoinLdsBytes = 81408;  // dynamic LDS per join workgroup: two workgroups share a CU's 160 KB
 constexpr int64_t kOutChunk = 16384;  // output pairs claimed per global allocation
 constexpr int kJoinGrid = 512;        // persistent join workgroups (2 per CU)
-constexpr int kPass2WgPerXcd = 16;    // pass-2 persistent workgroups per XCD and table (one per CU)
+constexpr int kPass2WgPerXcd = 16;    // pass-2 persistent workgroups per XCD, half of them (one per CU in all)
 constexpr int kPass2ItemTiles = 4;    // pass-2 items hold about this many full tiles
 constexpr int kMaxCombinedBits = 16;  // combined histogram limit (65536 partitions in LDS)
 constexpr int kMaxTotalBits = 24;     // two passes of at most 12 bits; above kMaxCombinedBits the
@@ -126,11 +126,13 @@ hipError_t launch_hist(const Layout& L, int key_bytes, hipStream_t s);
 hipError_t launch_colscan(const Layout& L, hipStream_t s);
 hipError_t launch_offsets(const Layout& L, hipStream_t s);
 hipError_t launch_pass1(const Layout& L, int key_bytes, hipStream_t s);
-hipError_t launch_pass2(const Layout& L, int key_bytes, hipStream_t s);
+// deep: the pass-2 digits were counted per item over pass 1's output
+// (launch_hist2, launch_segscan) instead of taken from the segment matrices.
+hipError_t launch_pass2(const Layout& L, int key_bytes, hipStream_t s, bool deep);
 // Deep plans: pass-2 digit counts per item over pass 1's output (h2, ipre),
 // their scan over each pass-1 partition's items and the fine totals (tot).
 hipError_t launch_hist2(const Layout& L, int key_bytes, hipStream_t s);
-hipError_t launch_segscan(const Layout& L, hipStream_t s);
+hipError_t launch_segscan(const Layout& L, int key_bytes, hipStream_t s);
 // Pass-2 items of a deep plan: at most this many per table.
 uint64_t deep_item_capacity(int64_t n, int key_bytes, const PartParams& pp);
 hipError_t launch_join_plan(const Layout& L, int base, int64_t slice, hipStream_t s);

@@ -33,7 +33,5 @@ size_t scan_ws_bytes(int64_t n);
 hipError_t scan_u32(const uint32_t* in, uint32_t* out, int64_t n, int inclusive, uint32_t* ws, hipStream_t s);
 hipError_t assign_blocks(const uint32_t* off, int64_t total, int P, int base, uint32_t* scanned, uint32_t* pidx,
                          int64_t max_blocks, uint32_t* d_total, uint32_t* ws, hipStream_t s);
-hipError_t p2_prep(const uint32_t* off1, int F1, uint32_t nseg, uint32_t* matc, uint32_t* mat_row0, int P,
-                   hipStream_t s);
 
 }  // namespace pj

@@ -382,23 +382,4 @@ hipError_t assign_blocks(const uint32_t* off, int64_t total, int P, int base, ui
   return hipGetLastError();
 }
 
-// ---------------------------------------------------------------------------
-// Pass-2 phase API set-up: treat the grouped input as the output of a single
-// pass-1 segment (matc row 0 = 0, rows >= 1 = partition sizes; mat row 0 = 0).
-// ---------------------------------------------------------------------------
-__global__ void k_p2_prep(const uint32_t* off1, int F1, uint32_t nseg, uint32_t* matc, uint32_t* mat_row0, int P) {
-  PJ_GRID_STRIDE(i, int64_t(nseg) * F1) {
-    const int64_t s = i / F1, p = i % F1;
-    matc[i] = s == 0 ? 0u : off1[p + 1] - off1[p];
-  }
-  PJ_GRID_STRIDE(q, P) mat_row0[q] = 0;
-}
-
-hipError_t p2_prep(const uint32_t* off1, int F1, uint32_t nseg, uint32_t* matc, uint32_t* mat_row0, int P,
-                   hipStream_t s) {
-  hipLaunchKernelGGL(k_p2_prep, dim3(grid_for(int64_t(nseg) * F1 + P, 256)), dim3(256), 0, s, off1, F1, nseg, matc,
-                     mat_row0, P);
-  return hipGetLastError();
-}
-
 }  // namespace pj

@@ -1056,6 +1056,12 @@ hipError_t launch_pass1(const Layout& L, int key_bytes, hipStream_t s) {
 // counts per run would give the XCD that holds a heavy key's partition all
 // of its items, each up to 256 times the size of an ordinary one.
 // ---------------------------------------------------------------------------
+// Items of a deep pass 2 at most: what h2 has room for (partition starts that
+// are not a partition of the n rows could ask for more).
+__host__ __device__ __forceinline__ uint32_t deep_items(uint32_t n, uint32_t chunk, int F1) {
+  return n / chunk + uint32_t(F1) + 1u;
+}
+
 __device__ __forceinline__ uint32_t p2_rank_to_p1(uint32_t r, uint32_t PX) { return (r % PX) * kNumXcd + r / PX; }
 
 template <int BLOCK, bool DEEP>
@@ -1073,7 +1079,8 @@ __device__ __forceinline__ void pass2_item_prefix(const PartTable& T, int F1, in
     nt[i] = 0;
     if (p1 < uint32_t(F1)) {
       if constexpr (DEEP) {
-        nt[i] = T.offc[p1 + 1] - T.offc[p1];
+        const uint32_t lo = min(T.offc[p1], T.n), hi = min(T.offc[p1 + 1], T.n);
+        nt[i] = hi > lo ? hi - lo : 0u;
         ng[i] = (nt[i] + chunk - 1) / chunk;
       } else {
         nt[i] = T.off[(p1 + 1) << b2] - T.off[p1 << b2];
@@ -1174,7 +1181,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
   // uniform keys).
   auto pre = [&](uint32_t r) { return uint32_t(__builtin_amdgcn_readfirstlane(s_pre[r])); };
   const uint32_t k_begin = uint32_t(__builtin_amdgcn_readfirstlane(s_run[0])) + uint32_t(j);
-  const uint32_t k_end = uint32_t(__builtin_amdgcn_readfirstlane(s_run[1]));
+  uint32_t k_end = uint32_t(__builtin_amdgcn_readfirstlane(s_run[1]));
+  if (DEEP) k_end = min(k_end, deep_items(T.n, chunk, F1));
   auto swap_counts = [&]() {
     uint32_t* t = s_cnt;
     s_cnt = s_cnt_next;
@@ -1203,7 +1211,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     uint32_t in_lo, in_hi, seg_lo = 0;
     if constexpr (DEEP) {
       in_lo = T.offc[p1] + g * chunk;
-      in_hi = min(in_lo + chunk, T.offc[p1 + 1]);
+      in_hi = min(min(in_lo + chunk, T.offc[p1 + 1]), T.n);
     } else {
       seg_lo = g * nseg / NG;
       const uint32_t seg_hi = (g + 1) * nseg / NG;
@@ -1283,11 +1291,11 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
   }
 }
 
-// Persistent pass-2 workgroups, kPass2WgPerXcd per XCD and table on average,
+// Persistent pass-2 workgroups, one per CU,
 // split between the tables by their sizes (the work is proportional to them):
 // the grid, and g0, the first workgroup of table 1 (a multiple of 8).
 static void pass2_grid(const Layout& L, uint32_t* grid, uint32_t* g0) {
-  const uint32_t per_xcd = uint32_t(kPass2WgPerXcd) * uint32_t(L.ntables);
+  const uint32_t per_xcd = uint32_t(kPass2WgPerXcd) * 2u;  // one table alone has all CUs
   uint32_t x0 = per_xcd;
   if (L.ntables > 1) {
     const double n0 = double(L.t[0].n), n1 = double(L.t[1].n);
@@ -1305,13 +1313,12 @@ static uint32_t pass2_chunk(int key_bytes, const PartParams& pp) {
 }
 
 uint64_t deep_item_capacity(int64_t n, int key_bytes, const PartParams& pp) {
-  return uint64_t(n) / pass2_chunk(key_bytes, pp) + uint64_t(pp.F1) + 1;
+  return deep_items(uint32_t(n), pass2_chunk(key_bytes, pp), pp.F1);
 }
 
-hipError_t launch_pass2(const Layout& L, int key_bytes, hipStream_t s) {
+hipError_t launch_pass2(const Layout& L, int key_bytes, hipStream_t s, bool deep) {
   uint32_t ngrid = 0, g0 = 0;
   pass2_grid(L, &ngrid, &g0);
-  const bool deep = L.pp.B > kMaxCombinedBits;
   dim3 grid(ngrid), block(kScatterBlock);
   // the item prefix (one entry per pass-1 partition rounded up to 8, plus one)
   // and the scan's temporaries follow the scatter's LDS
@@ -1373,7 +1380,7 @@ __global__ __launch_bounds__(BLOCK) void k_hist2(PartTable t0, PartTable t1, Par
   pass2_item_prefix<BLOCK, true>(T, F1, pp.b2, chunk, s_pre, s_tmp);
   if (local == 0)
     for (uint32_t r = tid; r <= RN; r += BLOCK) T.ipre[r] = s_pre[r];
-  const uint32_t n_items = s_pre[RN];
+  const uint32_t n_items = min(s_pre[RN], deep_items(T.n, chunk, F1));
   const tup_t* in = static_cast<const tup_t*>(T.buf1);
   for (uint32_t k = local; k < n_items; k += groups) {
     uint32_t lo = 0, hi = RN;  // s_pre[lo] <= k < s_pre[hi]
@@ -1382,10 +1389,20 @@ __global__ __launch_bounds__(BLOCK) void k_hist2(PartTable t0, PartTable t1, Par
       if (s_pre[mid] <= k) lo = mid; else hi = mid;
     }
     const uint32_t p1 = p2_rank_to_p1(lo, PX), g = k - s_pre[lo];
-    const uint32_t in_lo = T.offc[p1] + g * chunk, in_hi = min(in_lo + chunk, T.offc[p1 + 1]);
+    const uint32_t in_lo = T.offc[p1] + g * chunk, in_hi = min(min(in_lo + chunk, T.offc[p1 + 1]), T.n);
     for (int d = tid; d < F2; d += BLOCK) s_bins[d] = 0;
     lds_barrier();
-    for (uint32_t i = in_lo + tid; i < in_hi; i += BLOCK) atomicAdd(&s_bins[in[i].x & mask], 1u);
+    // eight keys a thread on their way together
+    constexpr uint32_t U = 8;
+    uint32_t i = in_lo + tid;
+    for (; i + (U - 1) * BLOCK < in_hi; i += U * BLOCK) {
+      uint32_t low[U];
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) low[u] = in[i + u * BLOCK].x;
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) atomicAdd(&s_bins[low[u] & mask], 1u);
+    }
+    for (; i < in_hi; i += BLOCK) atomicAdd(&s_bins[in[i].x & mask], 1u);
     lds_barrier();
     for (int d = tid; d < F2; d += BLOCK) T.h2[size_t(k) * F2 + d] = s_bins[d];
     lds_barrier();
@@ -1398,6 +1415,8 @@ hipError_t launch_hist2(const Layout& L, int key_bytes, hipStream_t s) {
   const uint32_t RN = uint32_t((L.pp.F1 + kNumXcd - 1) / kNumXcd) * kNumXcd;
   const size_t lds = (size_t(L.pp.F2) + RN + 1 + kScatterBlock / kWave + 1) * 4;
   const uint32_t chunk = pass2_chunk(key_bytes, L.pp);
+  ngrid *= 2;  // two workgroups share a CU
+  g0 *= 2;
   if (key_bytes == 4)
     hipLaunchKernelGGL((k_hist2<4, kScatterBlock>), dim3(ngrid), dim3(kScatterBlock), lds, s, L.t[0], L.t[1], L.pp,
                        chunk, g0);
@@ -1409,7 +1428,7 @@ hipError_t launch_hist2(const Layout& L, int key_bytes, hipStream_t s) {
 
 // One thread per fine partition q = p1 * F2 + d: the exclusive scan of digit
 // d's counts over p1's items (in place) and their total, tot[q].
-__global__ __launch_bounds__(256) void k_segscan(PartTable t0, PartTable t1, PartParams pp) {
+__global__ __launch_bounds__(256) void k_segscan(PartTable t0, PartTable t1, PartParams pp, uint32_t chunk) {
   const PartTable T = blockIdx.y ? t1 : t0;
   const uint32_t q = blockIdx.x * 256u + threadIdx.x;
   if (q >= uint32_t(pp.P)) return;
@@ -1417,7 +1436,8 @@ __global__ __launch_bounds__(256) void k_segscan(PartTable t0, PartTable t1, Par
   const uint32_t PX = uint32_t(pp.F1 + kNumXcd - 1) / kNumXcd;
   const uint32_t r = (p1 % kNumXcd) * PX + p1 / kNumXcd;
   uint32_t acc = 0;
-  for (uint32_t k = T.ipre[r]; k < T.ipre[r + 1]; ++k) {
+  const uint32_t k1 = min(T.ipre[r + 1], deep_items(T.n, chunk, pp.F1));
+  for (uint32_t k = T.ipre[r]; k < k1; ++k) {
     const uint32_t v = T.h2[size_t(k) * F2 + d];
     T.h2[size_t(k) * F2 + d] = acc;
     acc += v;
@@ -1425,8 +1445,9 @@ __global__ __launch_bounds__(256) void k_segscan(PartTable t0, PartTable t1, Par
   T.tot[q] = acc;
 }
 
-hipError_t launch_segscan(const Layout& L, hipStream_t s) {
-  hipLaunchKernelGGL(k_segscan, dim3((L.pp.P + 255) / 256, L.ntables), dim3(256), 0, s, L.t[0], L.t[1], L.pp);
+hipError_t launch_segscan(const Layout& L, int key_bytes, hipStream_t s) {
+  hipLaunchKernelGGL(k_segscan, dim3((L.pp.P + 255) / 256, L.ntables), dim3(256), 0, s, L.t[0], L.t[1], L.pp,
+                     pass2_chunk(key_bytes, L.pp));
   return hipGetLastError();
 }
 
