@@ -874,6 +874,12 @@ static hipError_t wide_join(const WideArgs& A, int key_bytes, int cfg, hipStream
 bool wide_shape(int64_t nR, int64_t nS, int key_bytes, WideShape* W) {
   const double n = double(nR);
   auto cap = [&](int cfg) { return (key_bytes == 4 ? kWideCfg4[cfg] : kWideCfg8[cfg]).cap(); };
+  // A scatter over 2048 digits costs less than one over 4096 (its runs are
+  // twice as long), so the large chunks come before the last doubling of the
+  // partitions: 20M x 90M int32 with payloads, 2048 partitions and chunks of
+  // 17408 in workgroups of a CU each: scatter 390 us, join 376; 4096 and
+  // chunks of 8704, two workgroups to a CU: 477 and 380.  16M x 64M int64:
+  // 437 + 516 against 520 + 475.
   int cfg, bits = 0;
   // 2^b partitions of at most `aim` build rows on average
   auto bits_for = [&](double aim, int least) {
@@ -887,16 +893,16 @@ bool wide_shape(int64_t nR, int64_t nS, int key_bytes, WideShape* W) {
     else if (nR <= int64_t(cap(4))) cfg = 4;
     else if (n <= 2048.0 * 512) { cfg = 0; bits = bits_for(2048.0, 6); }
     else if (n < 4096.0 * 2048) { cfg = 1; bits = bits_for(4096.0, 9); }
-    else if (n <= 8192.0 * 4096) { cfg = 2; bits = bits_for(8192.0, 11); }
-    else { cfg = 3; bits = 12; }
+    else if (n <= 8192.0 * 2048) { cfg = 2; bits = bits_for(8192.0, 11); }
+    else { cfg = 3; bits = n <= 16384.0 * 2048 ? 11 : 12; }
     if (n > 16384.0 * 4096) return false;
   } else {
     if (nR <= int64_t(cap(0))) cfg = 0;
     else if (nR <= int64_t(cap(1))) cfg = 1;
     else if (nR <= int64_t(cap(2))) cfg = 2;
     else if (n <= 1536.0 * 512) { cfg = 0; bits = bits_for(1536.0, 6); }
-    else if (n <= 4608.0 * 4096) { cfg = 1; bits = bits_for(4608.0, 9); }
-    else { cfg = 2; bits = 12; }
+    else if (n <= 4608.0 * 2048) { cfg = 1; bits = bits_for(4608.0, 9); }
+    else { cfg = 2; bits = n <= 9728.0 * 2048 ? 11 : 12; }
     if (n > 9728.0 * 4096) return false;
   }
   W->bits = bits;

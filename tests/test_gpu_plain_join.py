@@ -130,3 +130,17 @@ def test_large_builds_where_the_tag_identifies_the_key(pj, torch, nb, ns):
         assert pairs.shape[0] == int((pid < nb).sum())
         assert bool((ids[pairs[:, 0]] == pid[pairs[:, 1]]).all())
         assert torch.unique(pairs[:, 1]).numel() == pairs.shape[0]
+
+
+@pytest.mark.parametrize("dtype,nb", [("int32", 1 << 24), ("int32", (1 << 24) + 1), ("int32", 1 << 25), ("int64", 4608 * 2048),
+                                      ("int64", 4608 * 2048 + 1), ("int64", 9728 * 2048), ("int64", 9728 * 2048 + 1)])
+def test_large_builds_around_the_last_doublings_of_the_partitions(pj, torch, dtype, nb):
+    """2048 and 4096 partitions and their chunk sizes, average and largest."""
+    g = torch.Generator(device="cuda").manual_seed(nb)
+    ids = torch.randperm(nb, generator=g, device="cuda")
+    pid = torch.randint(0, 2 * nb, (1 << 22,), generator=g, device="cuda")
+    spread = (lambda x: (x * 0x2545F491).to(torch.int32)) if dtype == "int32" else (lambda x: x * 0x2545F4914F6CDD1D)
+    pairs = pj.partitioned_join(spread(ids), spread(pid)).to(torch.int64)
+    assert pairs.shape[0] == int((pid < nb).sum())
+    assert bool((ids[pairs[:, 0]] == pid[pairs[:, 1]]).all())
+    assert torch.unique(pairs[:, 1]).numel() == pairs.shape[0]
