@@ -29,8 +29,12 @@ namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// Tuples as vectors of their bytes (16-byte tuples as a native vector: arrays
-// of a struct type can end up in scratch memory).
+// Partitioned tuples: 8 bytes, or 12 with 8-byte keys (three words, loaded and
+// stored as one access each: the scatter of 16M x 64M rows takes 366 us and
+// the join 487; with a fourth, empty word they took 437 and 516).
+struct __attribute__((packed, aligned(4))) Tup12 {
+  uint32_t x, y, z;
+};
 template <int KB> struct WideTup;
 template <> struct WideTup<4> {
   using type = uint2;
@@ -39,13 +43,14 @@ template <> struct WideTup<4> {
   __device__ __forceinline__ static int32_t pay(const type& t) { return int32_t(t.y); }
 };
 template <> struct WideTup<8> {
-  using type = u32x4;
+  using type = Tup12;
   __device__ __forceinline__ static type make(uint64_t k, int32_t p) {
-    return type{uint32_t(k), uint32_t(k >> 32), uint32_t(p), 0u};
+    return type{uint32_t(k), uint32_t(k >> 32), uint32_t(p)};
   }
   __device__ __forceinline__ static uint64_t key(const type& t) { return uint64_t(t.x) | (uint64_t(t.y) << 32); }
   __device__ __forceinline__ static int32_t pay(const type& t) { return int32_t(t.z); }
 };
+constexpr size_t wide_tuple_bytes(int key_bytes) { return key_bytes == 4 ? 8 : 12; }
 
 __device__ __forceinline__ uint32_t wide_hash(uint32_t k) { return k * 0x9E3779B1u; }
 __device__ __forceinline__ uint32_t wide_hash(uint64_t k) {
@@ -878,8 +883,8 @@ bool wide_shape(int64_t nR, int64_t nS, int key_bytes, WideShape* W) {
   // twice as long), so the large chunks come before the last doubling of the
   // partitions: 20M x 90M int32 with payloads, 2048 partitions and chunks of
   // 17408 in workgroups of a CU each: scatter 390 us, join 376; 4096 and
-  // chunks of 8704, two workgroups to a CU: 477 and 380.  16M x 64M int64:
-  // 437 + 516 against 520 + 475.
+  // chunks of 8704, two workgroups to a CU: 477 and 380.  16M x 64M int64
+  // (tuples of 16 bytes then): 437 + 516 against 520 + 475.
   int cfg, bits = 0;
   // 2^b partitions of at most `aim` build rows on average
   auto bits_for = [&](double aim, int least) {
@@ -920,7 +925,7 @@ bool wide_shape(int64_t nR, int64_t nS, int key_bytes, WideShape* W) {
   uint64_t slice = (uint64_t(sl) + round - 1) / round * round;
   if (slice < round) slice = round;
   W->slice = uint32_t(slice < (1u << 20) ? slice : (1u << 20));
-  // Scatter tiles: 16 rows a thread (8 of 16-byte tuples), fewer when the
+  // Scatter tiles: 16 rows a thread (8 of 12-byte tuples), fewer when the
   // tables have too few rows to give every CU a few tiles.
   const int64_t rows = nR + nS;
   const int big = key_bytes == 4 ? 16 : 8;
@@ -931,15 +936,16 @@ bool wide_shape(int64_t nR, int64_t nS, int key_bytes, WideShape* W) {
 // Rows left free after each partition, so that partitions start an odd number
 // of 128-byte lines apart on average.
 static uint32_t wide_pad(int64_t n, int key_bytes, int bits) {
-  const uint32_t per_line = key_bytes == 4 ? 16 : 8;
-  const uint32_t lines = uint32_t((n >> bits) / per_line);
-  return (lines % 2 ? 4u : 5u) * per_line;
+  const uint32_t lines = uint32_t((uint64_t(n) >> bits) * wide_tuple_bytes(key_bytes) / 128);
+  // 16 tuples are a line of 8-byte tuples; 32 are three lines of 12-byte ones
+  if (key_bytes == 4) return (lines % 2 ? 4u : 5u) * 16;
+  return (lines % 2 ? 2u : 1u) * 32;
 }
 
 size_t wide_ws_bytes(int64_t nR, int64_t nS, int key_bytes, const WideShape& W) {
   if (W.bits == 0) return 0;
   auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
-  const size_t P = size_t(1) << W.bits, tb = key_bytes == 4 ? 8 : 16;
+  const size_t P = size_t(1) << W.bits, tb = wide_tuple_bytes(key_bytes);
   const size_t scan = (P + kWideScan - 1) / kWideScan * kWideScan;
   return up((size_t(nR) + P * wide_pad(nR, key_bytes, W.bits)) * tb) +
          up((size_t(nS) + P * wide_pad(nS, key_bytes, W.bits)) * tb) + 2 * up(P * 4) + up(scan * 4) + up((3 * kWideScanMax + 1) * 4) +
@@ -959,7 +965,7 @@ void wide_carve(int64_t nR, int64_t nS, int key_bytes, const WideShape& W, char*
     ws += (b + 255) & ~size_t(255);
     return p;
   };
-  const size_t P = size_t(1) << W.bits, tb = key_bytes == 4 ? 8 : 16;
+  const size_t P = size_t(1) << W.bits, tb = wide_tuple_bytes(key_bytes);
   A->pad[0] = wide_pad(nR, key_bytes, W.bits);
   A->pad[1] = wide_pad(nS, key_bytes, W.bits);
   A->tup[0] = take((size_t(nR) + P * A->pad[0]) * tb);
@@ -1000,7 +1006,7 @@ hipError_t launch_wide_scan(const WideArgs& A, hipStream_t s) {
 template <int KB, int E>
 static hipError_t wide_scatter_t(const WideArgs& A, hipStream_t s) {
   const uint32_t P = 1u << A.bits, tile = kWideBlock * E;
-  const size_t lds = size_t(tile) * (KB == 4 ? 8 : 16) + size_t(P) * 6 + 8;
+  const size_t lds = size_t(tile) * wide_tuple_bytes(KB) + size_t(P) * 6 + 8;
   const uint32_t nt = (A.n[0] + tile - 1) / tile + kNumXcd + (A.n[1] + tile - 1) / tile;
   uint32_t grid = lds * 2 <= 150 * 1024 ? 512u : 256u;
   if (nt < grid) grid = (nt + kNumXcd - 1) / kNumXcd * kNumXcd;
