@@ -1,6 +1,6 @@
 """Benchmark: radix-partitioned join of 64M unique int32 build keys with 256M
-int32 probe keys (50 % match), row-id payloads, two radix passes, on one
-MI355X.  One step = one full join (histogram, both partition passes, work list,
+int32 probe keys (50 % match), row-id payloads, on one
+MI355X.  One step = one full join (histogram, the partition passes, work list,
 LDS hash join, output compaction) with inputs resident in HBM.
 
 Prints one JSON line: whole-job tuples/s, the roofline of the dominant kernel

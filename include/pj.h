@@ -91,8 +91,8 @@ typedef struct pj_phase_times {
   float histogram_ms;   /* combined histogram of both tables (one key read)   */
   float offsets_ms;     /* column scans and partition offsets                 */
   float pass1_ms;       /* partition pass 1 (build + probe, one launch)       */
-  float pass2_ms;       /* partition pass 2 (build + probe, one launch)       */
-  float skew_ms;        /* join work list (block assignment)                  */
+  float pass2_ms;       /* partition pass 2 (build + probe, one launch); 0 if one pass sufficed */
+  float skew_ms;        /* join work list (block assignment); 0 if one pass sufficed */
   float join_ms;        /* build + probe of all partitions (one launch)       */
   float compact_ms;     /* output compaction after the join                   */
   float total_ms;       /* first event to last event                          */
@@ -110,6 +110,9 @@ const char* pj_last_error(void);
 /* Plain plan for a join of these tables (reads only n and key_bytes): the fewest radix bits whose
  * average build partition holds at most 2048 tuples (4-byte keys) or 1024 (8-byte keys), 1 pass
  * up to 2^10 partitions, else 2 passes (ceil / floor halves of the bits).
+ * A join with this plan, with or without the unique-key promise, or with a
+ * learned one may run in fewer passes and other partitions (same pairs, same
+ * workspace); a plan with other bits, factor or probe slice runs as it says.
  * Replaces the reference's hand-chosen -n/-N (main.cu:239-254). */
 pj_status pj_plan_default(const pj_table* build, const pj_table* probe, pj_plan* plan);
 

@@ -279,8 +279,8 @@ static void prof_recorded(bool one_pass = false) {
 // library chose the plan (it is the plain plan but for the unique-key promise,
 // or the learned planner's) and the build table is small enough.  Plans whose
 // caller chose the radix bits, chunk factor or probe slice are run as they
-// say.  64M x 256M int32: 3.36 ms in the plain plan's two passes, 2.59 ms in
-// one; 1M x 4M 176 against 103 us; 4K x 16K 111 against 44 us.  `need` is the
+// say.  64M x 256M int32: 3.31 ms in the plain plan's two passes, 2.3 ms in
+// one; 1M x 4M 176 against 102 us; 4K x 16K 110 against 41 us.  `need` is the
 // plan's workspace, whose last 256 bytes stay free.
 static bool wide_route(int64_t nR, int64_t nS, int key_bytes, const pj_plan& plan, size_t need, WideShape* W) {
   pj_plan plain;

@@ -98,6 +98,9 @@ constexpr int kWideBlock = 1024;  // histogram and scatter workgroup
 // k_wide_hist: rows are dealt to the XCD shares in tiles of `tile` rows (tile
 // t to share t % 8), as the scatter takes them.  Workgroups [0, g0) serve
 // table 0, the others table 1.  cnt[table][share][digit] is zero on entry.
+// Bound by reading the keys once: 64M x 256M int32 211 us, 1.34 GB at 6.4 TB/s
+// (257 us before, with one workgroup to a CU and a [segment][digit] matrix to
+// write); two workgroups a CU need its bins at 16 KB each.
 // ---------------------------------------------------------------------------
 template <int KB, bool VEC>
 __global__ __launch_bounds__(kWideBlock) void k_wide_hist(WideArgs A, uint32_t g0) {
@@ -179,7 +182,8 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_hist(WideArgs A, uint32_t g
 // 16 blocks): start[table][digit] and cnt[table][share][digit], which becomes
 // the share's write cursor, are relative to the block.  The join's items of a
 // partition are its build chunks times its probe slices.  Also clears the pair
-// count.
+// count.  A latency chain of a few loads: 5 us at 4096 digits (the column and
+// offset scans it stands for took 37 us at 64M x 256M).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kWideScan) void k_wide_scan(WideArgs A) {
   __shared__ uint32_t s_tmp[3][kWideScan / kWave + 1];
@@ -241,6 +245,15 @@ __device__ __forceinline__ void block_prefixes(const WideArgs& A, uint32_t (*s_p
 // and stored.  The runs of one tile are a few tuples long, but the tiles of
 // an XCD fill the same lines one after another within its L2, which writes
 // them back whole.
+// Bound by memory, and by what its writes add to it: 64M x 256M 1.19 ms for
+// 1.34 GB read and 2.68 GB of tuples, of which 3.45 GB reach memory (each
+// atomic writes its line of cursors through, and some lines leave the L2
+// unfinished at 4096 digits); the two passes it stands for took 2.19 ms.  The
+// cost of a digit count on random keys, 256M tuples: 512 digits 0.69 ms, 2048
+// 0.74, 4096 0.92.  16K-tuple tiles: runs of 4 tuples at 4096 digits; tiles of
+// 8K with two workgroups to a CU were slower, and so were claims after the
+// staging (1223 -> 1295 us) and stores kept back until the next tile's staging
+// (1441 us).  The cursor adds of two digits at once: 1223 -> 1205 us.
 // ---------------------------------------------------------------------------
 template <int KB, int E, bool PAY>
 __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_wide_scatter(WideArgs A) {
@@ -440,6 +453,14 @@ __device__ __forceinline__ uint32_t zero_bytes(uint32_t x) {
 // during the next round, whose probes hide the claim.  A round in which some
 // probe matches twice walks its buckets again to write them.
 // COLS: no partitions (bits == 0): both sides are read from the key columns.
+// Bound by memory under many probes a build row (16M x 256M Zipf: 4.3 GB in
+// 1.02 ms, 4.2 TB/s, against 0.94 ms in smaller tables before), otherwise by
+// the build of an item, about 17 us for 16384 tuples with nothing else on the
+// CU (64M x 256M: 0.94 ms, of which 0.27 the builds; with walks of
+// {key, payload} entries in place of the tags 1.68 ms).  Repeated build keys
+// are bound by the walks and the uncoalesced stores of their rounds: 12M x 24M
+// with keys four times 414 us, of which 230 those two; their pairs read a
+// window at a time took registers that spilled (64M x 256M 1.24 ms).
 template <int KB, int BLOCK, int NB, int U, int LGB, bool VERIFY, bool COLS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_wide_join(WideArgs A) {
   using key_t = typename KeyT<KB>::key_t;
@@ -891,7 +912,15 @@ bool wide_shape(int64_t nR, int64_t nS, int key_bytes, WideShape* W) {
   // chunks of 8704, two workgroups to a CU: 477 and 380.  16M x 64M int64
   // (tuples of 16 bytes then): 437 + 516 against 520 + 475.
   int cfg, bits = 0;
-  // 2^b partitions of at most `aim` build rows on average
+  // 2^b partitions of at most `aim` build rows on average.  No partitions
+  // while one chunk holds the table: 3072 x 12288 int32 20 us, 6144 x 24576
+  // 21 us, and with 12288 x 49152 at 30 us the line is reached (12289 rows in
+  // 64 partitions 29 us).  The larger chunk takes over where the partitions
+  // double otherwise: 1M x 4M 87 us with chunks of 3072, one row more with
+  // 6144 74; 8M x 32M 328 on both sides of the line where the keys leave the
+  // table.  Past the last line the two-pass pipeline: 67.1M x 134M int32
+  // 1.74 ms here, one row more 2.40 ms there; 39.8M x 79.7M int64 1.51 and
+  // 2.55 ms.
   auto bits_for = [&](double aim, int least) {
     int b = least;
     while (n / double(1 << b) > aim) ++b;
@@ -919,8 +948,8 @@ bool wide_shape(int64_t nR, int64_t nS, int key_bytes, WideShape* W) {
   W->cfg = cfg;
   W->cap = cap(cfg);
   // Probe slices: every slice builds its chunk's table again, so a slice has
-  // at least four times the average chunk's rows, unless the items would not
-  // fill the chip.
+  // eight times the average chunk's rows, unless the items would not fill the
+  // chip (1024 of them).
   const uint32_t round = uint32_t((key_bytes == 4 ? kWideCfg4[cfg] : kWideCfg8[cfg]).block * (key_bytes == 4 ? 8 : 6));
   const double chunk = n / double(1 << bits);
   double sl = 8.0 * chunk, fill = double(nS) / 1024.0;
@@ -931,7 +960,8 @@ bool wide_shape(int64_t nR, int64_t nS, int key_bytes, WideShape* W) {
   if (slice < round) slice = round;
   W->slice = uint32_t(slice < (1u << 20) ? slice : (1u << 20));
   // Scatter tiles: 16 rows a thread (8 of 12-byte tuples), fewer when the
-  // tables have too few rows to give every CU a few tiles.
+  // tables have too few rows to give every CU a few tiles (a tile's digits
+  // cost the same whatever its rows: 1M x 4M in tiles of 4K, 64M in 16K).
   const int64_t rows = nR + nS;
   const int big = key_bytes == 4 ? 16 : 8;
   W->rows_per_thread = rows >= int64_t(512) * kWideBlock * big ? big : rows >= int64_t(512) * kWideBlock * big / 2 ? big / 2 : big / 4;
@@ -939,7 +969,9 @@ bool wide_shape(int64_t nR, int64_t nS, int key_bytes, WideShape* W) {
 }
 
 // Rows left free after each partition, so that partitions start an odd number
-// of 128-byte lines apart on average.
+// of 128-byte lines apart on average: the open lines of evenly filled
+// partitions are otherwise in the same sets of the L2 (scatter of 64M x 256M
+// 1340 us without, 1223 with).
 static uint32_t wide_pad(int64_t n, int key_bytes, int bits) {
   const uint32_t lines = uint32_t((uint64_t(n) >> bits) * wide_tuple_bytes(key_bytes) / 128);
   // 16 tuples are a line of 8-byte tuples; 32 are three lines of 12-byte ones
